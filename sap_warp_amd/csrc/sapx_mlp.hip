@@ -243,6 +243,14 @@ __host__ __device__ __forceinline__ int act_offset(const LayerOffsets& lo, int l
     for (int i = 0; i < l; ++i) off += rows * (lo.dims[i] + kRowPad);
     return off;
 }
+// inference keeps two layers at a time: the even ones share one buffer, the odd ones the other behind
+// it, so the two never take more than all layers together (one wide layer among narrow ones: two
+// buffers of the widest would)
+__host__ __device__ __forceinline__ int widest(const LayerOffsets& lo, int parity) {
+    int w = 0;
+    for (int l = parity; l <= lo.L; l += 2) w = lo.dims[l] > w ? lo.dims[l] : w;
+    return w;
+}
 
 // CT tiles of 16 columns starting at tile t0, MT tiles of 16 rows: acc = act . W^T over `steps` pairs
 // of MFMA column groups (act: LDS rows of stride ls; Wp: packed weights).  The weights of U steps are
@@ -366,9 +374,8 @@ __global__ __launch_bounds__(kWaves * 64) void row_block_kernel(RowBlockArgs g) 
     const int r0 = blockIdx.x * R;
     const int L = g.lo.L;
     // inference needs two layers' activations at a time, training keeps them all
-    int wmax = 0;
-    for (int l = 0; l <= L; ++l) wmax = g.lo.dims[l] > wmax ? g.lo.dims[l] : wmax;
-    auto act = [&](int l) { return sm + (TRAIN ? act_offset(g.lo, l, R) : (l & 1) * R * (wmax + kRowPad)); };
+    const int odd = TRAIN ? 0 : R * (widest(g.lo, 0) + kRowPad);
+    auto act = [&](int l) { return sm + (TRAIN ? act_offset(g.lo, l, R) : (l & 1) * odd); };
     {
         const int d0 = g.lo.dims[0], ls = d0 + kRowPad;
         const float* mean = g.norm;
@@ -820,10 +827,10 @@ struct SapxMlp {
         return c;
     }
     size_t train_lds(int mt) const { return (size_t)act_offset(lo, lo.L + 1, 16 * mt) * 2; }
-    size_t forward_lds(int mt) const { return (size_t)2 * 16 * mt * (maxw() + kRowPad) * 2; }
+    size_t forward_lds(int mt) const { return (size_t)16 * mt * (widest(lo, 0) + widest(lo, 1) + 2 * kRowPad) * 2; }
 };
 
-// all layers' activations of 16 rows fit in the LDS of a workgroup
+// all layers' activations of 16 rows fit in the LDS of a workgroup (then two buffers of the forward pass do)
 static bool net_fits(const SapxMlp* M) { return M->train_lds(1) <= kMaxLds; }
 
 static int32_t reserve(SapxMlp* M, int batch) {

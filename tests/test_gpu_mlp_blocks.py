@@ -1,8 +1,10 @@
 """The warm-start network's kernels at the edges of their row blocks, against the numpy restatement
 with the same bfloat16 rounding points (oracle/learned_oracle.py): one row, ragged rows of a 16-row
 block, the first batch in 32-row blocks, one, two and three hidden layers of widths that give the
-waves one, two and four column tiles, an output wider than a tile, and a network too wide for the row
-blocks (one GEMM per layer)."""
+waves one, two and four column tiles, an output wider than a tile, one wide layer among narrow ones up
+to the widest that the row blocks take (4864 between 128 inputs and 64 outputs), where two buffers of the
+widest layer would exceed a workgroup's LDS from 2560 on, and networks too wide for the row blocks (one
+GEMM per layer)."""
 from __future__ import annotations
 
 import numpy as np
@@ -18,6 +20,13 @@ pytestmark = pytest.mark.gpu
     (17, 64, 70, (256, 128)),
     (100, 311, 35, (512, 512, 512)),
     (4097, 200, 20, (192, 128)),
+    (33, 70, 9, (2496,)),
+    (4097, 70, 9, (2560,)),
+    (33, 311, 35, (2560, 512)),
+    (65, 311, 35, (512, 3072)),
+    (20, 311, 35, (4096,)),
+    (33, 70, 9, (4864,)),
+    (33, 70, 9, (4928,)),
     (33, 70, 9, (5120,)),
 ])
 def test_mlp_row_blocks_match_oracle(gpu_device, rows, features, outputs, hidden):
