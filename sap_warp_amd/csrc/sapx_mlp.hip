@@ -788,12 +788,12 @@ struct SapxMlp {
     uint16_t* dz[2] = {nullptr, nullptr};
     uint16_t* dzt[2] = {nullptr, nullptr};
     // a network that runs on row blocks: packed transposed activations (ht) and gradients, the row
-    // blocks' bias gradients and losses; its forward pass needs no workspace
+    // blocks' bias gradients and losses, and y for outputs that overlap their input (other forward
+    // passes need no workspace)
     bool row_blocks = false;
     uint16_t* dzp[kMaxLayers] = {nullptr};
     float* bias_part = nullptr;
     float* loss_part = nullptr;
-    size_t y_cap = 0;  // bytes of y where it only serves overlapping outputs
     void free_ws() {
         void* ps[] = {xb, xt, y, dz[0], dz[1], dzt[0], dzt[1], bias_part, loss_part};
         for (void* p : ps)
@@ -807,7 +807,6 @@ struct SapxMlp {
         xb = xt = nullptr;
         y = bias_part = loss_part = nullptr;
         dz[0] = dz[1] = dzt[0] = dzt[1] = nullptr;
-        y_cap = 0;
         cap = 0;
     }
     ~SapxMlp() {
@@ -846,6 +845,7 @@ static int32_t reserve(SapxMlp* M, int batch) {
         }
         MLP_HIP(hipMalloc(&M->bias_part, (size_t)(Bp / 16) * M->bias_cols() * 4));
         MLP_HIP(hipMalloc(&M->loss_part, (size_t)(Bp / 16) * 4));
+        MLP_HIP(hipMalloc(&M->y, (size_t)Bp * M->out_features * 4));
         M->cap = Bp;
         return SAPX_OK;
     }
@@ -1055,17 +1055,14 @@ int32_t sapx_mlp_forward(SapxMlp* M, const float* x, int32_t batch, float* y, vo
     if (M->row_blocks) {
         RowBlockArgs a = row_block_args(M, x, batch);
         a.Bp = (batch + 15) / 16 * 16;
-        // an output that overlaps the input goes through a buffer: a block writes its rows of y while
+        // an output that overlaps the input goes through the workspace: a block writes its rows of y while
         // others still read theirs of x
         const size_t out_bytes = (size_t)batch * M->out_features * 4;
         const uintptr_t xa = (uintptr_t)x, ya = (uintptr_t)y;
         const bool overlap = ya < xa + (size_t)batch * M->in_features * 4 && xa < ya + out_bytes;
-        if (overlap && M->y_cap < out_bytes) {
-            if (M->y) (void)hipFree(M->y);
-            M->y = nullptr;
-            M->y_cap = 0;
-            MLP_HIP(hipMalloc(&M->y, out_bytes));
-            M->y_cap = out_bytes;
+        if (overlap) {
+            const int32_t rc = reserve(M, batch);
+            if (rc != SAPX_OK) return rc;
         }
         a.y = overlap ? M->y : y;
         // Blocks of 16 rows while that gives each of the 256 CUs at most one (4096 rows: 21 us; 20 us

@@ -82,3 +82,31 @@ def test_mlp_row_blocks_match_oracle(gpu_device, rows, features, outputs, hidden
     over[:rows * features].copy_(xd.reshape(-1))
     m.forward(over[:rows * features].view(rows, features), over[:rows * outputs].view(rows, outputs))
     assert bool((over[:rows * outputs].view(rows, outputs) == want).all())
+
+
+def test_captured_overlapping_forward(gpu_device):
+    """A forward pass onto its own input, captured on a reserved workspace (nothing is allocated then):
+    every replay gives what the pass gives eagerly, also with eager passes between them."""
+    import torch
+
+    from sap_warp_amd.learned import Mlp
+
+    rows, features, outputs = 70, 64, 20
+    m = Mlp(features, outputs, hidden=(128, 192), seed=5, out_scale=1.0)
+    m.reserve(rows)
+    buf = torch.zeros(rows * features, dtype=torch.float32, device="cuda:0")
+    x, y = buf.view(rows, features), buf[:rows * outputs].view(rows, outputs)
+    want = torch.empty((rows, outputs), dtype=torch.float32, device="cuda:0")
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            m.forward(x, y)
+        gen = torch.Generator(device="cuda:0").manual_seed(2)
+        for _ in range(4):
+            rand = torch.randn((rows, features), generator=gen, device="cuda:0")
+            m.forward(rand, want)
+            buf.copy_(rand.reshape(-1))
+            g.replay()
+            stream.synchronize()
+            assert torch.equal(y, want)
