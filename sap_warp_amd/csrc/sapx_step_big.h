@@ -225,15 +225,17 @@ __device__ __forceinline__ void solve(float* H, int npad, const unsigned* hm, fl
         const f4 s = (a[0] * x[0] + a[1] * x[1]) + (a[2] * x[2] + a[3] * x[3]);
         return (s[0] + s[1]) + (s[2] + s[3]);
     };
-    // r -= sum_t a[t] y_t, y_t on lane t of every row of 16 lanes
-    auto take = [&](const f4 (&a)[4], float y) {
+    // r -= sum_t a[t] y_t on the lanes that `use` it, y_t on lane t of every row of 16 lanes; the wave's
+    // lanes stay together while they read others' y
+    auto take = [&](bool use, const f4 (&a)[4], float y) {
+        if (!__any(use)) return;
         float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
         for (int t = 0; t < kB; t += 2) {
             s0 = fmaf(a[t >> 2][t & 3], rl(y, t), s0);
             s1 = fmaf(a[(t + 1) >> 2][(t + 1) & 3], rl(y, t + 1), s1);
         }
-        r -= s0 + s1;
+        r -= use ? s0 + s1 : 0.0f;
     };
     f4 Y[4], p[4], x[4];
     for (int kb = 0; kb < nblk; ++kb) {
@@ -248,7 +250,7 @@ __device__ __forceinline__ void solve(float* H, int npad, const unsigned* hm, fl
         __syncthreads();
         sixteen(xr + kB * kb, x);
         const float y = dot(Y, x);
-        if (use) take(p, y);
+        take(use, p, y);
         if (ib == kb) r = y;
         if (ib == kb + 1 && live) xr[tid] = r;
     }
@@ -271,7 +273,7 @@ __device__ __forceinline__ void solve(float* H, int npad, const unsigned* hm, fl
         __syncthreads();
         sixteen(xr + kB * kb, x);
         const float y = dot(Y, x);
-        if (use) take(p, y);
+        take(use, p, y);
         if (ib == kb) r = y;
         if (ib == kb - 1) xr[tid] = r;
     }
