@@ -7,6 +7,9 @@ struct SapxModel;
 
 namespace sapx {
 
+constexpr int kCus = 256;              // compute units of the chip
+constexpr size_t kLdsGrain = 1280;     // allocation unit of a workgroup's LDS
+
 // LDS layout of the one-wave-per-world step kernel (byte offsets); js / ls are
 // the row strides of the contact Jacobian and of the dynamics matrix (NP + 4:
 // rows start on 16 bytes and a column group of 16 rows falls on different banks).

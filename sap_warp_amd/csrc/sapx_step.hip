@@ -2183,12 +2183,15 @@ hipError_t launch_step(const StepParams& P, hipStream_t stream) {
         attr_set = true;
     }
     const dim3 grid(P.m.W), block(NT);
-    // Three workgroups a CU where the LDS of three fits: 168 registers then, with more of the set-up's
-    // values spilled, but a third more worlds in flight (687 worlds of 16 bodies, 96 dofs: 4.11 -> 3.36 ms).
-    // Where only two fit the spills are all that is left of it (128 worlds of 32 bodies: 4.58 -> 4.75 ms).
+    // Three workgroups a CU where the LDS of three fits and there are worlds for a third one: 168 registers
+    // then, with more of the set-up's values spilled, but a third more worlds in flight (687 worlds of 16
+    // bodies, 96 dofs: 4.11 -> 3.36 ms).  Where only two share a CU the spills are all that is left of it (128
+    // worlds of 32 bodies: 4.58 -> 4.75 ms).
+    const size_t lds = (P.smem_bytes + kLdsGrain - 1) / kLdsGrain * kLdsGrain;
+    const bool three = 3 * lds <= 160 * 1024 && P.m.W > 2 * kCus;
     if (!P.g_work) hipLaunchKernelGGL((sapx_step_kernel<NT, kMatricesLds, 2>), grid, block, P.smem_bytes, stream, P);
     else if (!P.hessian_lds) hipLaunchKernelGGL((sapx_step_kernel<NT, kMatricesGlobal, 2>), grid, block, P.smem_bytes, stream, P);
-    else if (3 * P.smem_bytes <= 160 * 1024) hipLaunchKernelGGL((sapx_step_kernel<NT, kHessianLds, 3>), grid, block, P.smem_bytes, stream, P);
+    else if (three) hipLaunchKernelGGL((sapx_step_kernel<NT, kHessianLds, 3>), grid, block, P.smem_bytes, stream, P);
     else hipLaunchKernelGGL((sapx_step_kernel<NT, kHessianLds, 2>), grid, block, P.smem_bytes, stream, P);
     return hipGetLastError();
 }

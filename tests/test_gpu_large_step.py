@@ -24,3 +24,35 @@ def test_block_edges(gpu_device, monkeypatch, bodies, slots, preset, ls):
     monkeypatch.setattr(step, "_scene", lambda name, worlds, seed: (
         hetero.build_pile_scene(worlds, seed=seed + 5, bodies=bodies, device="cuda:0"), 2.0e-3, slots))
     step._run_and_compare(f"pile of {bodies}", preset, ls, worlds=2, steps=2, warm_steps=120, min_max_contacts=bodies)
+
+
+def test_builds_agree(gpu_device):
+    """More than 512 worlds whose LDS lets three share a CU run in the build with fewer registers: the
+    first worlds of such a batch end where they end in a batch of two, up to what another order of float32
+    operations moves a refined solve (each build is within 1e-5 of the oracle)."""
+    import numpy as np
+    import torch
+
+    from sap_warp_amd import hetero
+    from sap_warp_amd.collision import SapCollisionPipeline
+    from sap_warp_amd.solver_sap import SolverSAP
+    from tests.helpers import world_rel_err
+
+    ends = []
+    for worlds in (2, 513):
+        model = hetero.build_pile_scene(worlds, seed=8, bodies=11, device="cuda:0")
+        solver = SolverSAP(model, max_rigid_contact=88, line_search_variant="exact_root", contact_preset_variant="approx32")
+        pipe = SapCollisionPipeline(model, max_contacts_per_world=88)
+        contacts = pipe.contacts()
+        s0, s1, control = model.state(), model.state(), model.control()
+        for _ in range(3):
+            pipe.collide(s0, contacts)
+            solver.step(s0, s1, control, contacts, 2.0e-3)
+            s0, s1 = s1, s0
+        torch.cuda.synchronize()
+        assert int(contacts.rigid_contact_world_start[2]) > 0
+        ends.append([getattr(s0, k)[:size].cpu().numpy().astype(np.float64).reshape(2, -1)
+                     for k, size in (("joint_q", 2 * 77), ("joint_qd", 2 * 66))])
+    for a, b in zip(*ends):
+        for w in range(2):
+            assert world_rel_err(b[w], a[w]) <= 2.0e-5, w
