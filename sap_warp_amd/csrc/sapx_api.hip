@@ -80,6 +80,7 @@ struct SapxModel {
     std::vector<int> h_shape_world, h_shape_type;  // host copies for pipeline set-up
     std::vector<float> h_shape_scale;
     int32_t world_count = 0, joint_count = 0, dof_count = 0, coord_count = 0, body_count = 0, shape_count = 0;
+    int row_dofs = 0;  // most dofs on the root paths of two bodies of a world
     ~SapxModel() {
         for (void* p : owned) (void)hipFree(p);
     }
@@ -101,10 +102,11 @@ struct SapxSolver {
     int npad = 0, js = 0, ast = 0;
     int lds[18] = {0};
     int smem_bytes = 0;
-    // large worlds: A, H and J of every world in device memory (fused kernel), floats
+    // large worlds (fused kernel): each world's block of device memory, offsets in floats (H lies in LDS
+    // where it fits)
     float* big_ws = nullptr;
     size_t big_stride = 0, big_A = 0, big_H = 0, big_J = 0, big_tmp = 0, big_ck = 0, big_rows = 0, big_cols = 0;
-    int hessian_lds = 0;
+    int hessian_lds = 0, row_dofs = 0;
     // one-wave-per-world kernel: LDS layouts of the contact variants (16 / 32 / 64 slots; a
     // variant whose layout does not fit has bytes == 0) and the current schedule
     bool wave_ok = false;
@@ -367,6 +369,16 @@ int32_t sapx_model_create(const SapxModelDesc* d, SapxModel** out) {
             j = p >= 0 ? body_joint[p] : -1;
         }
     }
+    // the longest contact row: the dofs on the root paths of two bodies
+    auto path_dofs = [&](unsigned long long joints) {
+        int dofs = 0;
+        for (; joints; joints &= joints - 1) dofs += t_jds[__builtin_ctzll(joints) + 1] - t_jds[__builtin_ctzll(joints)];
+        return dofs;
+    };
+    int row_dofs = 0;
+    if (NB <= 64)  // the step kernels' worlds
+        for (int a = 0; a < NB; ++a)
+            for (int b = 0; b <= a; ++b) row_dofs = std::max(row_dofs, path_dofs(anc[a] | anc[b]));
     // child-body lists (CSR) for the deterministic reverse-level composite sweep
     std::vector<int> child_start(NB + 1, 0), child_list;
     for (int c = 0; c < NB; ++c) {
@@ -461,6 +473,7 @@ int32_t sapx_model_create(const SapxModelDesc* d, SapxModel** out) {
     m->h_shape_world.assign(d->shape_world, d->shape_world + Stot);
     m->h_shape_type.assign(d->shape_type, d->shape_type + Stot);
     m->h_shape_scale.assign(d->shape_scale, d->shape_scale + 3 * (size_t)Stot);
+    m->row_dofs = row_dofs;
     dm.W = W; dm.J = J; dm.N = N; dm.NQ = NQ; dm.NB = NB; dm.S = S;
     dm.P = (int)per_world[0].size() / 2;
     dm.num_levels = nlev;
@@ -730,8 +743,10 @@ int32_t sapx_solver_create(const SapxModel* model, const SapxSolverOpts* opts, S
         s->big_J = region(j_bytes);
         s->big_tmp = region((size_t)C * 104);
         s->big_ck = region((size_t)C * 14 * 8);
-        s->big_rows = region((size_t)(n * (size_t)C + 1) / 2 * 4 + (size_t)3 * n * C * 4);
-        s->big_cols = region((size_t)(npad * (size_t)C + 1) / 2 * 4 + (size_t)3 * npad * C * 4);
+        s->row_dofs = model->row_dofs;
+        const size_t entries = (size_t)s->row_dofs * C;  // of the contact rows, by contact and by dof
+        s->big_rows = region((entries + 1) / 2 * 4 + 3 * entries * 4);
+        s->big_cols = region((entries + 1) / 2 * 4 + 3 * entries * 4);
         s->big_H = s->hessian_lds ? 0 : region(packed);
         s->big_stride = at;
         const size_t bytes = (size_t)dm.W * s->big_stride * sizeof(float);
@@ -1038,6 +1053,7 @@ static int32_t fill_step_params(SapxSolver* s, const SapxStateView* in, const Sa
     P.g_rows = s->big_rows;
     P.g_cols = s->big_cols;
     P.hessian_lds = s->hessian_lds;
+    P.row_dofs = s->row_dofs;
     P.o_bx = s->lds[17];
     return SAPX_OK;
 }

@@ -80,6 +80,7 @@ struct StepParams {
     size_t g_stride;
     size_t g_A, g_H, g_J, g_tmp, g_ck, g_rows, g_cols;
     int hessian_lds;
+    int row_dofs;        // most dofs on the root paths of two bodies: the longest contact row
     int o_bx;            // LDS: block masks and solve buffer of a large world
     WaveLayout wl;       // one-wave kernel layout for this launch's contact variant
     int wave_min_nc;     // the variant processes worlds with wave_min_nc <= nc <= its capacity

@@ -483,7 +483,7 @@ struct BigWorld {
     int lo = 0, hi = 0;        // columns of A that this thread's dof (row) can touch: its tree's
     unsigned* am = nullptr;    // LDS: blocks of A, blocks of the factor (row masks)
     unsigned* hm = nullptr;
-    float* buf = nullptr;      // LDS: 32 floats of the solves
+    float* buf = nullptr;      // LDS: npad floats of the solves
 };
 
 // (A x) of this thread's dof: A is symmetric, so neighbouring threads read neighbouring words of row j
@@ -1414,29 +1414,27 @@ __global__ __launch_bounds__(NT, WGS) void sapx_step_kernel(StepParams P) {
     int parity = 0;
     if constexpr (BIG) {
         // ---- contact rows by contact and by dof: the dofs on the root paths of a contact's two bodies,
-        // slot-major so that neighbouring threads read neighbouring words
+        // slot-major so that neighbouring threads read neighbouring words.  By contact a slot holds every
+        // contact; by dof only those that have as many entries, the dofs with more of them first: slot l
+        // starts at sum_d min(count_d, l).  Both then take row_dofs C entries (a dense list by dof took n C:
+        // 2.17 instead of 0.88 MB a world of 32 bodies and 256 contacts).
+        const size_t entries = (size_t)P.row_dofs * C;
         float* g = P.g_work + (size_t)blockIdx.x * P.g_stride;
         unsigned short* rl_idx = reinterpret_cast<unsigned short*>(g + P.g_rows);
-        float* rl_val = g + P.g_rows + ((size_t)n * C + 1) / 2;
+        float* rl_val = g + P.g_rows + (entries + 1) / 2;
         unsigned short* cl_idx = reinterpret_cast<unsigned short*>(g + P.g_cols);
-        float* cl_val = g + P.g_cols + ((size_t)npad * C + 1) / 2;
+        float* cl_val = g + P.g_cols + (entries + 1) / 2;
         double* vel = s.ck + (size_t)C * kCk;  // contacts past the first NT: vc, dvc
         int* packed = reinterpret_cast<int*>(s.tmp);
+        int* starts = packed + C;
+        int* counts = reinterpret_cast<int*>(bw.buf);  // contacts of each dof
         auto path = [&](int c) {
             const int b0 = s.cb[c * 2], b1 = s.cb[c * 2 + 1];
             return (b0 >= 0 ? T.body_anc[b0] : 0ull) | (b1 >= 0 ? T.body_anc[b1] : 0ull);
         };
-        int cl_count = 0;
-        if (tid < n) {
-            const int ji = T.dof_joint[tid];
-            for (int c = 0; c < nc; ++c) {
-                if (!bit(path(c), ji)) continue;
-                cl_idx[(size_t)cl_count * npad + tid] = (unsigned short)c;
-#pragma unroll
-                for (int r = 0; r < 3; ++r) cl_val[((size_t)r * C + cl_count) * npad + tid] = s.J[(c * 3 + r) * js + tid];
-                ++cl_count;
-            }
-        }
+        if (tid < npad) counts[tid] = 0;
+        if (tid < big::kMaxBlocks) bw.hm[tid] = bw.am[tid];
+        __syncthreads();
         for (int c = tid; c < nc; c += NT) {
             int k = 0;
             unsigned blocks = 0u;
@@ -1445,19 +1443,43 @@ __global__ __launch_bounds__(NT, WGS) void sapx_step_kernel(StepParams P) {
                 for (int d = T.jds[j]; d < T.jds[j + 1]; ++d) {
                     rl_idx[(size_t)k * C + c] = (unsigned short)d;
 #pragma unroll
-                    for (int r = 0; r < 3; ++r) rl_val[((size_t)r * n + k) * C + c] = s.J[(c * 3 + r) * js + d];
+                    for (int r = 0; r < 3; ++r) rl_val[((size_t)r * P.row_dofs + k) * C + c] = s.J[(c * 3 + r) * js + d];
+                    atomicAdd(counts + d, 1);
                     blocks |= 1u << (d >> 4);
                     ++k;
                 }
             }
             packed[c] = (int)(blocks | ((unsigned)k << 16));
         }
-        if (tid < big::kMaxBlocks) bw.hm[tid] = bw.am[tid];
         __syncthreads();
+        int cl_count = 0, rank = 0;
+        if (tid < n) {
+            cl_count = counts[tid];
+            for (int d = 0; d < n; ++d) rank += counts[d] > cl_count || (counts[d] == cl_count && d < tid);
+        }
+        for (int c = tid; c < nc; c += NT) {
+            int start = 0;
+            for (int d = 0; d < n; ++d) start += min(counts[d], c);
+            starts[c] = start;
+        }
+        __syncthreads();
+        if (tid < n) {
+            const int ji = T.dof_joint[tid];
+            int l = 0;
+            for (int c = 0; c < nc; ++c) {
+                if (!bit(path(c), ji)) continue;
+                const size_t e = (size_t)starts[l++] + rank;
+                cl_idx[e] = (unsigned short)c;
+#pragma unroll
+                for (int r = 0; r < 3; ++r) cl_val[r * entries + e] = s.J[(c * 3 + r) * js + tid];
+            }
+        }
+        __syncthreads();
+        // s.cb: blocks of the contact's row and their dof count (upper half); start of a slot by dof
         for (int c = tid; c < nc; c += NT) {
             const unsigned p = (unsigned)packed[c], blocks = p & 0xffffu;
-            s.cb[c * 2] = (int)blocks;
-            s.cb[c * 2 + 1] = (int)(p >> 16);
+            s.cb[c * 2] = (int)p;
+            s.cb[c * 2 + 1] = starts[c];
             for (unsigned m = blocks; m; m &= m - 1) {
                 const int ib = __builtin_ctz(m);
                 atomicOr(bw.hm + ib, blocks & ((2u << ib) - 1u));
@@ -1472,8 +1494,8 @@ __global__ __launch_bounds__(NT, WGS) void sapx_step_kernel(StepParams P) {
             for (int k = 0; k < count; ++k) {
                 const double xv = x[rl_idx[(size_t)k * C + c]];
                 s0 += (double)rl_val[(size_t)k * C + c] * xv;
-                s1 += (double)rl_val[((size_t)n + k) * C + c] * xv;
-                s2 += (double)rl_val[((size_t)2 * n + k) * C + c] * xv;
+                s1 += (double)rl_val[entries + (size_t)k * C + c] * xv;
+                s2 += (double)rl_val[2 * entries + (size_t)k * C + c] * xv;
             }
             out[0] = s0; out[1] = s1; out[2] = s2;
         };
@@ -1482,10 +1504,11 @@ __global__ __launch_bounds__(NT, WGS) void sapx_step_kernel(StepParams P) {
             double s0 = 0.0, s1 = 0.0, s2 = 0.0;
 #pragma unroll 4
             for (int l = 0; l < cl_count; ++l) {
-                const double* y = s.cv + 3 * (int)cl_idx[(size_t)l * npad + tid];
-                s0 += (double)cl_val[(size_t)l * npad + tid] * y[0];
-                s1 += (double)cl_val[((size_t)C + l) * npad + tid] * y[1];
-                s2 += (double)cl_val[((size_t)2 * C + l) * npad + tid] * y[2];
+                const size_t e = (size_t)s.cb[2 * l + 1] + rank;
+                const double* y = s.cv + 3 * (int)cl_idx[e];
+                s0 += (double)cl_val[e] * y[0];
+                s1 += (double)cl_val[entries + e] * y[1];
+                s2 += (double)cl_val[2 * entries + e] * y[2];
             }
             return (s0 + s1) + s2;
         };
@@ -1495,7 +1518,7 @@ __global__ __launch_bounds__(NT, WGS) void sapx_step_kernel(StepParams P) {
         if (tid < nc) {
 #pragma unroll
             for (int k = 0; k < kCk; ++k) k8[k] = s.ck[(size_t)tid * kCk + k];
-            count0 = s.cb[2 * tid + 1];
+            count0 = s.cb[2 * tid] >> 16;
         }
         auto contacts = [&](auto&& f) {
             if (tid < nc) f(tid, k8, vc0, dvc0, count0);
@@ -1508,7 +1531,7 @@ __global__ __launch_bounds__(NT, WGS) void sapx_step_kernel(StepParams P) {
                     a[r] = vel[(size_t)6 * c + r];
                     b[r] = vel[(size_t)6 * c + 3 + r];
                 }
-                f(c, kk, a, b, s.cb[2 * c + 1]);
+                f(c, kk, a, b, s.cb[2 * c] >> 16);
 #pragma unroll
                 for (int r = 0; r < 3; ++r) {
                     vel[(size_t)6 * c + r] = a[r];

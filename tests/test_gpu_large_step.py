@@ -26,6 +26,14 @@ def test_block_edges(gpu_device, monkeypatch, bodies, slots, preset, ls):
     step._run_and_compare(f"pile of {bodies}", preset, ls, worlds=2, steps=2, warm_steps=120, min_max_contacts=bodies)
 
 
+@pytest.mark.parametrize("preset,ls", [("approx32", "exact_root"), ("drake", "armijo_decay")])
+def test_articulated(gpu_device, preset, ls):
+    """Contact rows over the joints of two root paths of one tree, so that the dofs' lists differ in
+    length: lying humanoids (35 dofs) with so many slots that J exceeds the LDS layout."""
+    step._run_and_compare("humanoid_lying", preset, ls, worlds=3, steps=2, warm_steps=50, solver_C=300, pipe_C=64,
+                          min_max_contacts=25)
+
+
 def test_builds_agree(gpu_device):
     """More than 512 worlds whose LDS lets three share a CU run in the build with fewer registers: the
     first worlds of such a batch end where they end in a batch of two, up to what another order of float32
@@ -56,3 +64,23 @@ def test_builds_agree(gpu_device):
     for a, b in zip(*ends):
         for w in range(2):
             assert world_rel_err(b[w], a[w]) <= 2.0e-5, w
+
+
+def test_block_of_device_memory(gpu_device):
+    """A world of 32 free bodies with 256 contact slots takes no more device memory than its dense A, H
+    and J (0.89 MB): the contact rows are listed by contact and by dof without their zeros."""
+    import torch
+
+    from sap_warp_amd import hetero
+    from sap_warp_amd.solver_sap import SolverSAP
+
+    worlds, n, slots = 128, 192, 256
+    model = hetero.build_pile_scene(worlds, seed=8, bodies=32, device="cuda:0")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    solver = SolverSAP(model, max_rigid_contact=slots, line_search_variant="exact_root", contact_preset_variant="approx32")
+    used = before - torch.cuda.mem_get_info()[0]
+    solver.close()
+    dense = 4 * (2 * n * (n + 1) + 3 * slots * (n + 1))
+    # outside the block: states, warm start and statistics of a world
+    assert used <= worlds * (dense + 50_000), (used / worlds, dense)
