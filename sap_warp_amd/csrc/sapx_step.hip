@@ -2206,12 +2206,14 @@ hipError_t launch_step(const StepParams& P, hipStream_t stream) {
         attr_set = true;
     }
     const dim3 grid(P.m.W), block(NT);
-    // Three workgroups a CU where the LDS of three fits and there are worlds for a third one: 168 registers
-    // then, with more of the set-up's values spilled, but a third more worlds in flight (687 worlds of 16
-    // bodies, 96 dofs: 4.11 -> 3.36 ms).  Where only two share a CU the spills are all that is left of it (128
-    // worlds of 32 bodies: 4.58 -> 4.75 ms).
+    // Three workgroups a CU where the LDS of three fits and they take the worlds in fewer rounds: 168
+    // registers then, with more of the set-up's values spilled, but a third more worlds in flight (600 worlds
+    // of 16 bodies, 96 dofs: 3.69 -> 3.03 ms; 600 humanoids with 300 slots: 1.01 -> 0.90 ms).  In as many
+    // rounds the spills are all that is left of it (512 such piles 2.66 -> 2.94 ms, 1000 of the humanoids 1.39 ->
+    // 1.45 ms).
     const size_t lds = (P.smem_bytes + kLdsGrain - 1) / kLdsGrain * kLdsGrain;
-    const bool three = 3 * lds <= 160 * 1024 && P.m.W > 2 * kCus;
+    auto rounds = [&](int share) { return (P.m.W + share * kCus - 1) / (share * kCus); };
+    const bool three = 3 * lds <= 160 * 1024 && rounds(3) < rounds(2);
     if (!P.g_work) hipLaunchKernelGGL((sapx_step_kernel<NT, kMatricesLds, 2>), grid, block, P.smem_bytes, stream, P);
     else if (!P.hessian_lds) hipLaunchKernelGGL((sapx_step_kernel<NT, kMatricesGlobal, 2>), grid, block, P.smem_bytes, stream, P);
     else if (three) hipLaunchKernelGGL((sapx_step_kernel<NT, kHessianLds, 3>), grid, block, P.smem_bytes, stream, P);
