@@ -486,12 +486,14 @@ struct BigWorld {
     float* buf = nullptr;      // LDS: npad floats of the solves
 };
 
-// (A x) of this thread's dof: A is symmetric, so neighbouring threads read neighbouring words of row j
+// (A x) of this thread's dof: A is symmetric, so neighbouring threads read neighbouring words of row j.
+// Bound by the latency of the loads, 16 of them under way at a time: a tree of 35 dofs takes three waits
+// instead of five with eight (8 humanoids with 300 slots 514 -> 507 us a step).
 __device__ __forceinline__ double row_times(const float* A, int ast, const BigWorld& bw, const double* x) {
     const float* a = A + threadIdx.x;
     double s0 = 0.0, s1 = 0.0;
     int j = bw.lo;
-#pragma unroll 4
+#pragma unroll 8
     for (; j + 1 < bw.hi; j += 2) {
         s0 += (double)a[(size_t)j * ast] * x[j];
         s1 += (double)a[(size_t)(j + 1) * ast] * x[j + 1];
@@ -1425,33 +1427,40 @@ __global__ __launch_bounds__(NT, WGS) void sapx_step_kernel(StepParams P) {
         unsigned short* cl_idx = reinterpret_cast<unsigned short*>(g + P.g_cols);
         float* cl_val = g + P.g_cols + (entries + 1) / 2;
         double* vel = s.ck + (size_t)C * kCk;  // contacts past the first NT: vc, dvc
-        int* packed = reinterpret_cast<int*>(s.tmp);
-        int* starts = packed + C;
+        unsigned long long* paths = reinterpret_cast<unsigned long long*>(s.tmp);  // joints of a contact's row
         int* counts = reinterpret_cast<int*>(bw.buf);  // contacts of each dof
-        auto path = [&](int c) {
-            const int b0 = s.cb[c * 2], b1 = s.cb[c * 2 + 1];
-            return (b0 >= 0 ? T.body_anc[b0] : 0ull) | (b1 >= 0 ? T.body_anc[b1] : 0ull);
-        };
         if (tid < npad) counts[tid] = 0;
         if (tid < big::kMaxBlocks) bw.hm[tid] = bw.am[tid];
         __syncthreads();
+        // both lists first by index, so that the loads of J behind them do not wait for each other
         for (int c = tid; c < nc; c += NT) {
-            int k = 0;
+            const int b0 = s.cb[c * 2], b1 = s.cb[c * 2 + 1];
+            unsigned long long m = (b0 >= 0 ? T.body_anc[b0] : 0ull) | (b1 >= 0 ? T.body_anc[b1] : 0ull);
+            paths[c] = m;
+            int count = 0;
             unsigned blocks = 0u;
-            for (unsigned long long m = path(c); m; m &= m - 1) {
+            for (; m; m &= m - 1) {
                 const int j = __builtin_ctzll(m);
                 for (int d = T.jds[j]; d < T.jds[j + 1]; ++d) {
-                    rl_idx[(size_t)k * C + c] = (unsigned short)d;
-#pragma unroll
-                    for (int r = 0; r < 3; ++r) rl_val[((size_t)r * P.row_dofs + k) * C + c] = s.J[(c * 3 + r) * js + d];
+                    rl_idx[(size_t)count++ * C + c] = (unsigned short)d;
                     atomicAdd(counts + d, 1);
                     blocks |= 1u << (d >> 4);
-                    ++k;
                 }
             }
-            packed[c] = (int)(blocks | ((unsigned)k << 16));
+#pragma unroll 4
+            for (int k = 0; k < count; ++k) {
+                const int d = rl_idx[(size_t)k * C + c];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) rl_val[r * entries + (size_t)k * C + c] = s.J[(c * 3 + r) * js + d];
+            }
+            s.cb[c * 2] = (int)(blocks | ((unsigned)count << 16));  // of the contact's row
+            for (unsigned left = blocks; left; left &= left - 1) {
+                const int ib = __builtin_ctz(left);
+                atomicOr(bw.hm + ib, blocks & ((2u << ib) - 1u));
+            }
         }
         __syncthreads();
+        if (tid < 64) big::symbolic(bw.hm, npad >> 4);
         int cl_count = 0, rank = 0;
         if (tid < n) {
             cl_count = counts[tid];
@@ -1460,37 +1469,28 @@ __global__ __launch_bounds__(NT, WGS) void sapx_step_kernel(StepParams P) {
         for (int c = tid; c < nc; c += NT) {
             int start = 0;
             for (int d = 0; d < n; ++d) start += min(counts[d], c);
-            starts[c] = start;
+            s.cb[c * 2 + 1] = start;  // of slot c of the list by dof
         }
         __syncthreads();
         if (tid < n) {
             const int ji = T.dof_joint[tid];
             int l = 0;
-            for (int c = 0; c < nc; ++c) {
-                if (!bit(path(c), ji)) continue;
-                const size_t e = (size_t)starts[l++] + rank;
-                cl_idx[e] = (unsigned short)c;
+#pragma unroll 4
+            for (int c = 0; c < nc; ++c)
+                if (bit(paths[c], ji)) cl_idx[(size_t)s.cb[2 * l++ + 1] + rank] = (unsigned short)c;
+#pragma unroll 4
+            for (l = 0; l < cl_count; ++l) {
+                const size_t e = (size_t)s.cb[2 * l + 1] + rank;
+                const int c = cl_idx[e];
 #pragma unroll
                 for (int r = 0; r < 3; ++r) cl_val[r * entries + e] = s.J[(c * 3 + r) * js + tid];
             }
         }
-        __syncthreads();
-        // s.cb: blocks of the contact's row and their dof count (upper half); start of a slot by dof
-        for (int c = tid; c < nc; c += NT) {
-            const unsigned p = (unsigned)packed[c], blocks = p & 0xffffu;
-            s.cb[c * 2] = (int)p;
-            s.cb[c * 2 + 1] = starts[c];
-            for (unsigned m = blocks; m; m &= m - 1) {
-                const int ib = __builtin_ctz(m);
-                atomicOr(bw.hm + ib, blocks & ((2u << ib) - 1u));
-            }
-        }
-        __syncthreads();
-        if (tid < 64) big::symbolic(bw.hm, npad >> 4);
-        // J x of contact c over its dofs
+        // J x of contact c over its dofs, the 12 of two free bodies in two waits (687 worlds of 16
+        // bodies 3044 us; in three 3151 us, eight dofs at a time 3059 us)
         auto rows_times = [&](const double* x, int c, int count, double* out) {
             double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-#pragma unroll 4
+#pragma unroll 6
             for (int k = 0; k < count; ++k) {
                 const double xv = x[rl_idx[(size_t)k * C + c]];
                 s0 += (double)rl_val[(size_t)k * C + c] * xv;
