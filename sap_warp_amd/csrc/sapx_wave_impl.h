@@ -463,7 +463,7 @@ __device__ __forceinline__ void wave_body(const StepParams& P, const int blk) {
     double* ck = reinterpret_cast<double*>(smem_raw + L.o_ck);    // slots x kCk
     float* cG = reinterpret_cast<float*>(smem_raw + L.o_cG);      // slots x 9
     float* Jm = reinterpret_cast<float*>(smem_raw + L.o_J);       // 3 slots x js
-    float* Lt = reinterpret_cast<float*>(smem_raw + L.o_Lt);      // NP x ls (+64)
+    float* Lt = reinterpret_cast<float*>(smem_raw + L.o_Lt);      // lower 16 x 16 blocks of the factor, 256 floats each
     float* Am = reinterpret_cast<float*>(smem_raw + L.o_A);       // n x ls dynamics matrix rows
     const float* arow = Am + (lane < n ? lane : 0) * ls;
     // kinematics scratch overlays the J / Lt region (phases 2-4 and 9)

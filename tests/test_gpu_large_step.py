@@ -1,9 +1,8 @@
 """Steps of worlds beyond the LDS layout: packed Newton matrix, contact rows listed by contact and dof.
 
 The 256-thread kernel against the float64 oracle where its blocks and loops have their edges: a last
-block of two dofs, full blocks only, the largest order (16 blocks, Newton matrix in device memory), the
-largest that keeps it in LDS with two and with three workgroups a CU, and more contact slots than
-threads.  Bars as for every step: 1e-5 in the velocities, the formed problem and the public state, which
+block of two dofs, full blocks only, the largest order (16 blocks, Newton matrix in device memory), a
+Newton matrix in LDS, and more contact slots than threads.  Bars as for every step: 1e-5 in the velocities, the formed problem and the public state, which
 float32 matrices of these scenes keep with two digits to spare (the solve is refined in float64)."""
 import pytest
 
