@@ -70,3 +70,35 @@ def test_unrefined_error(gpu_device, n):
     error = unrefined_error(n, 10)
     print(f"chol n {n} unrefined error {error:.3e}", flush=True)
     assert error <= 4.1e-7
+
+
+def test_solves_on_several_streams(gpu_device):
+    """Two handles whose solves each fill the chip (512 workgroups, two a CU) on a stream each, and a third
+    of another size beside them: every solve ends where it ends alone, bit for bit, and none times out."""
+    import torch
+
+    from sap_warp_amd.blocked_cholesky import BlockCholeskySolverBatched
+
+    rng = np.random.default_rng(3)
+    handles = []
+    for n, batch in ((200, 128), (512, 64), (1100, 12)):
+        A = torch.tensor(np.stack([_spd(n, rng) for _ in range(2)]), device="cuda:0").repeat(batch // 2, 1, 1)
+        rhs = torch.tensor(rng.normal(size=(batch, n)), device="cuda:0")
+        solver = BlockCholeskySolverBatched(n, batch, refine=2)
+        solver.factorize(A, n)
+        alone = torch.zeros_like(rhs)
+        solver.solve(rhs, alone)
+        assert np.all(solver.info() == 0)
+        ref = torch.linalg.solve(A[:2].double().cpu(), rhs[:2].cpu())
+        assert float((alone[:2].cpu() - ref).abs().max()) <= 1e-10 * float(ref.abs().max())
+        handles.append((solver, rhs, alone, torch.zeros_like(rhs), torch.cuda.Stream()))
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for solver, rhs, _, x, stream in handles:
+            with torch.cuda.stream(stream):
+                solver.solve(rhs, x)
+    torch.cuda.synchronize()
+    for solver, _, alone, x, _ in handles:
+        assert np.all(solver.info() == 0)
+        assert torch.equal(x, alone)
+        solver.close()
