@@ -16,8 +16,8 @@
 // solved by 16 x 16 blocks of which only those that a tree, a contact or fill touches exist
 // (sapx_step_big.h).  Bound by the latency of that chain of phases at one or a few worlds a CU.  Measured
 // against dense matrices in device memory with a row or a column per wave: 687 worlds of 16 bodies
-// (96 dofs, 128 contact slots, 27 iterations at most) 9.6 -> 3.36 ms, 128 worlds of 32 bodies (192 dofs,
-// 256 slots, 35 iterations) 24.1 -> 4.6 ms.
+// (96 dofs, 128 contact slots, 27 iterations at most) 9.6 -> 2.85 ms, 128 worlds of 32 bodies (192 dofs,
+// 256 slots, 35 iterations) 24.1 -> 4.15 ms.
 //
 // Precision: kinematics, dynamics, the contact Jacobian, the Hessian and its
 // Cholesky factor are float32 (the reference's approx32 preset solves its
@@ -2208,9 +2208,9 @@ hipError_t launch_step(const StepParams& P, hipStream_t stream) {
     const dim3 grid(P.m.W), block(NT);
     // Three workgroups a CU where the LDS of three fits and they take the worlds in fewer rounds: 168
     // registers then, with more of the set-up's values spilled, but a third more worlds in flight (600 worlds
-    // of 16 bodies, 96 dofs: 3.69 -> 3.03 ms; 600 humanoids with 300 slots: 1.01 -> 0.90 ms).  In as many
-    // rounds the spills are all that is left of it (512 such piles 2.66 -> 2.94 ms, 1000 of the humanoids 1.39 ->
-    // 1.45 ms).
+    // of 16 bodies, 96 dofs: 3.45 -> 2.82 ms; 600 humanoids with 300 slots: 0.94 -> 0.87 ms).  In as many
+    // rounds the spills are all that is left of it (512 such piles 2.20 -> 2.54 ms, 1000 of the humanoids 1.32 ->
+    // 1.36 ms).
     const size_t lds = (P.smem_bytes + kLdsGrain - 1) / kLdsGrain * kLdsGrain;
     auto rounds = [&](int share) { return (P.m.W + share * kCus - 1) / (share * kCus); };
     const bool three = 3 * lds <= 160 * 1024 && rounds(3) < rounds(2);
