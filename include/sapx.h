@@ -348,7 +348,8 @@ typedef struct SapxSchedule {
     int32_t kernel;         /* SAPX_KERNEL_*                                                   */
     int32_t small_capacity; /* wave: contact slots (16, 32 or 64) that the variant for the
                                worlds with the fewest contacts has at least; larger variants
-                               take the others                                                  */
+                               take the others (worlds that are all on the chip at once with
+                               slots for every contact take one launch)                         */
     int32_t fork;           /* wave: launch the larger variants on a second stream beside it    */
     int32_t world_order;    /* wave: dispatch worlds most-expensive-first                       */
 } SapxSchedule;

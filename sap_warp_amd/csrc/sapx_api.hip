@@ -112,6 +112,8 @@ struct SapxSolver {
     bool wave_ok = false;
     WaveLayout wl16{}, wl32{}, wl64{};
     WaveLayout wl_four{}, wl_three{};  // the most slots (<= 64) with four / three worlds a CU
+    WaveLayout wl_all{};               // the fewest slots that hold every contact
+    int wave_resident = 0;             // worlds on the chip at once in that layout
     SapxSchedule sched{};
     // the variants above the first run on a second stream (default priority), forked from and joined
     // back into the caller's stream, so their few long worlds overlap the first one's launch
@@ -806,6 +808,9 @@ int32_t sapx_solver_create(const SapxModel* model, const SapxSolverOpts* opts, S
             };
             s->wl_four = shared(4);
             s->wl_three = shared(3);
+            s->wl_all = fit((C + 3) / 4 * 4);
+            if (s->wl_all.bytes)  // four: what the registers allow
+                s->wave_resident = kCus * std::min<int>(4, 160 * 1024 / (int)round_up(s->wl_all.bytes, kLdsGrain));
             // the 64-slot variant holds every world; the small ones need it beside them when C > slots
             s->wave_ok = s->wl64.bytes > 0 || (C <= 16 && s->wl16.bytes > 0) || (C <= 32 && s->wl32.bytes > 0);
         }
@@ -1085,17 +1090,26 @@ int32_t sapx_step(SapxSolver* s, const SapxStateView* in, const SapxStateView* o
         }
         // contact variants: each world runs in the smallest that holds it.  LDS decides how many worlds
         // share a CU, so the first variant has the most slots that leave room for four (what the registers
-        // allow; the schedule's slots if those are more), the second for three, the last is the 64-slot one.
+        // allow; the schedule's slots if those are more), the second for three, the last holds every contact.
         // Steps with 16 and 64 slots against these: 2069 piles of 8 bodies, 48 dofs and 20 contacts (24, 40
         // and 64 slots) 1463 -> 1090 us, 4096 humanoids, a third of them lying with 22-34 contacts, 934 -> 815
         // us.  A stream for each variant was slower for the piles (1138 us): the blocks of the 64-slot launch
         // that have no world hold LDS while they pass.
+        // Where all worlds are on the chip at once in the layout for every contact, smaller ones let no more
+        // of them run, and the launches of a stream follow each other, the worlds with the most contacts last:
+        // one launch (512 worlds of convex bodies, 54 dofs and 32 slots, Armijo: 790 -> 432 us, and 741 us with
+        // 16 and 64 slots; 64 quadrupeds with 64 slots 194 -> 185 us, 510 piles of 8 bodies 658 -> 636 us).
         std::vector<const WaveLayout*> run;
         const int small = s->sched.small_capacity;
         run.push_back(small == 16 ? &s->wl16 : (small == 32 ? &s->wl32 : &s->wl64));
-        if (s->wl_four.slots > small && run[0]->slots < P.C) run[0] = &s->wl_four;
-        for (const WaveLayout* L : {&s->wl_three, &s->wl64})
-            if (run.back()->slots < P.C && L->slots > run.back()->slots) run.push_back(L);
+        if (run[0]->slots < P.C) {
+            const bool resident = (int)dm.W <= s->wave_resident;
+            if (resident || s->wl_four.slots >= s->wl_all.slots) run[0] = &s->wl_all;
+            else if (s->wl_four.slots > small) run[0] = &s->wl_four;
+            if (run[0]->slots < P.C && s->wl_three.slots > run[0]->slots && s->wl_three.slots < s->wl_all.slots)
+                run.push_back(&s->wl_three);
+            if (run.back()->slots < P.C) run.push_back(&s->wl_all);
+        }
         auto launch_run = [&](size_t k, hipStream_t sq) {
             StepParams Q = P;
             Q.wl = *run[k];

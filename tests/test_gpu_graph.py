@@ -1,5 +1,5 @@
-"""The whole step (collision + solver step, with the forked 64-contact launch and the
-dispatch-order kernel) captured in a HIP graph and replayed: every replay must equal the
+"""The whole step (collision + solver step with the dispatch-order kernel; 8 worlds take one launch, 520
+are forked over the contact variants) captured in a HIP graph and replayed: every replay must equal the
 eager step from the same input, with eager work and synchronisations between replays.
 """
 from __future__ import annotations
@@ -14,14 +14,15 @@ def _np(t):
     return t.detach().cpu().numpy()
 
 
-def test_graph_replay_matches_eager(gpu_device):
+@pytest.mark.parametrize("worlds", [8, 520])
+def test_graph_replay_matches_eager(gpu_device, worlds):
     import torch
 
     from sap_warp_amd.collision import SapCollisionPipeline
     from sap_warp_amd.scenes import build_humanoid_scene
     from sap_warp_amd.solver_sap import SolverSAP
 
-    model = build_humanoid_scene(8, seed=3, device="cuda:0")
+    model = build_humanoid_scene(worlds, seed=3, device="cuda:0")
     solver = SolverSAP(model, max_rigid_contact=64, line_search_variant="exact_root")
     pipe = SapCollisionPipeline(model, max_contacts_per_world=64)
     contacts = pipe.contacts()

@@ -26,18 +26,19 @@ def test_block_edges(gpu_device, monkeypatch, bodies, slots):
                           min_max_contacts=1)
 
 
-@pytest.mark.parametrize("lying,slots", [(1.0, 64), (0.5, 30)])
-def test_contact_variants_agree(gpu_device, lying, slots):
+@pytest.mark.parametrize("lying,slots,worlds", [(1.0, 64, 24), (0.5, 30, 24), (1.0, 64, 520), (0.5, 30, 1040)])
+def test_contact_variants_agree(gpu_device, lying, slots, worlds):
     """Worlds split over the contact variants of a step (fewest contacts first, on two streams or on one)
     end where the 64-slot variant alone takes them: a variant is a choice of LDS layout, the arithmetic
-    and its order are the same, so the states are equal bit for bit."""
+    and its order are the same, so the states are equal bit for bit.  24 worlds fit on the chip at once and
+    take one launch whatever the schedule; 520 with 64 slots (three launches) and 1040 with 32 (two) do not."""
     import torch
 
     from sap_warp_amd.collision import SapCollisionPipeline
     from sap_warp_amd.scenes import build_humanoid_scene
     from sap_warp_amd.solver_sap import SolverSAP
 
-    model = build_humanoid_scene(24, seed=4, lying_fraction=lying, contact_gap=0.05, device="cuda:0")
+    model = build_humanoid_scene(worlds, seed=4, lying_fraction=lying, contact_gap=0.05, device="cuda:0")
     ends = []
     for small, fork in ((64, False), (16, True), (16, False), (32, True)):
         solver = SolverSAP(model, max_rigid_contact=slots, line_search_variant="exact_root",
