@@ -349,7 +349,9 @@ def test_ant_step_parity(gpu_device):
 
 @pytest.mark.parametrize("small,fork,order", [(32, True, True), (32, False, False), (16, False, True)])
 def test_humanoid_step_parity_schedules(gpu_device, small, fork, order):
-    """Other work schedules of the wave kernel (32-slot variant, serial variants, identity order)."""
+    """Other work schedules of the wave kernel against the oracle.  Six worlds fit on the chip at once and
+    take one launch under each of them (in the order given); test_contact_variants_agree compares the
+    variants and streams of a split batch with that launch, bit for bit."""
     _run_and_compare("humanoid", "drake", "exact_root", worlds=6, steps=3,
                      schedule={"kernel": "wave", "small_capacity": small, "fork": fork, "world_order": order})
 
